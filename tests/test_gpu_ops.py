@@ -1,5 +1,7 @@
 """Operator parity on the device: each ernie_hip op against the oracle and the
 reference's own known-answer tests (ported in kat.py)."""
+import math
+
 import numpy as np
 import pytest
 
@@ -116,6 +118,32 @@ def test_gemm_fp32_split_products(ctx, m, n, k, ldc):
     c = empty((m, ldc)).fill_(float("nan"))
     ctx.gemm(dev(a), k, dev(w), k, c, ldc, m, n, k, E.FP32, E.FP32)
     assert np.all(np.abs(host(c)[:, :n] - a64 @ w64.T) <= (k + 1) * 2.0**-24 * (np.abs(a64) @ np.abs(w64).T))
+
+
+@pytest.mark.parametrize("m,n,k", [(130, 140, 48), (33, 260, 4096)])
+@pytest.mark.parametrize("sa,sw", [(1e-36, 1.0), (1.0, 1e-37), (1e-37, 1e30), (1e-42, 1e20), (1e-20, 1e-15)])
+def test_gemm_fp32_small_magnitudes(ctx, m, n, k, sa, sw):
+    # Values down to FP32 subnormals keep all their bits. Error of a sum of k products
+    # in FP32: at most k 2^-24 of sum |a| |w|, about sqrt(k) 2^-24 of it in the 2-norm, where
+    # |result| is about sum |a| |w| / sqrt(k): k 2^-24 at the very most, and about 2e-7
+    # measured; lost low bits of a value of 1e-36 alone give 2.6e-5.
+    a, w = O.normal((m, k), 3) * np.float32(sa), O.normal((n, k), 4) * np.float32(sw)
+    ref = a.astype(np.float64) @ w.astype(np.float64).T
+    c = empty((m, n)).fill_(float("nan"))
+    ctx.gemm(dev(a), k, dev(w), k, c, n, m, n, k, E.FP32, E.FP32)
+    assert np.linalg.norm(host(c) - ref) <= 1e-6 * np.linalg.norm(ref)
+
+
+def test_gemm_fp32_identity_returns_every_value(ctx):
+    # Values of all exponents with random significands, subnormals included, times the
+    # identity: the parts of each value add up to it exactly.
+    m, k = 4096, 32
+    rng = np.random.default_rng(11)
+    bits = (np.arange(m * k, dtype=np.uint32) % 255) << 23 | rng.integers(0, 1 << 23, m * k, dtype=np.uint32)
+    a = (bits | rng.integers(0, 2, m * k, dtype=np.uint32) << 31).view(np.float32).reshape(m, k)
+    c = empty((m, k))
+    ctx.gemm(dev(a), k, dev(np.eye(k, dtype=np.float32)), k, c, k, m, k, k, E.FP32, E.FP32)
+    assert np.array_equal(host(c), a)
 
 
 def test_gemm_fp32_infinities_and_the_largest_values(ctx):
@@ -405,3 +433,39 @@ def test_sdpa_fp32_split_products_and_infinities(ctx, d, sq, sk):
     assert np.all(np.isposinf(got[1, :, d - 1]))
     got[1, :, d - 1] = ref[1, :, d - 1]
     assert np.abs(got - ref).max() <= bound
+
+
+def sdpa_reference(q, k, v):
+    s = np.einsum("hqd,hkd->hqk", q.astype(np.float64), k.astype(np.float64)) / np.sqrt(q.shape[-1])
+    p = np.exp(s - s.max(-1, keepdims=True))
+    return np.einsum("hqk,hkd->hqd", p / p.sum(-1, keepdims=True), v.astype(np.float64))
+
+
+@pytest.mark.parametrize("sq,sk,sv,scale", [(1e-36, 1e36, 1.0, 1.0), (1e36, 1e-36, 1e-36, 1.0), (1.0, 1.0, 1e-37, 1.0),
+                                            (1e-20, 1e20, 1e25, 1.0), (1e15, 1e15, 1.0, 1e-30)])
+def test_sdpa_fp32_small_magnitudes(ctx, sq, sk, sv, scale):
+    # Queries, keys, values and a scale near the ends of FP32: the relative error is that of
+    # values near 1 (4e-7 measured), where parts of BF16 subnormals would give 2.6e-5 and more.
+    n, d = 130, 128
+    q, k, v = (O.normal((2, n, d), i) * np.float32(x) for i, x in ((7, sq), (8, sk), (9, sv)))
+    out = empty((2, n, d)).fill_(float("nan"))
+    st = (n * d, d) * 4
+    ctx.sdpa(dev(q), dev(k), dev(v), out, E.FP32, 2, 2, n, n, d, st, scale=scale / math.sqrt(d))
+    ref = sdpa_reference(q.astype(np.float64) * scale, k, v)
+    assert np.linalg.norm(host(out) - ref) <= 2e-6 * np.linalg.norm(ref)
+
+
+def test_sdpa_fp32_small_probabilities(ctx):
+    # A first key with all the weight and no value, others with probabilities of about 1e-37
+    # and values of 1e30. A score near -120 in log2 units is rounded to 2^-18 of a unit
+    # and scaled and subtracted once each: 1e-5 of a probability at most; parts that end at
+    # 2^-133 would lose 2^-134 / 2^-123, 5e-4 of it.
+    n, d = 70, 64
+    q, k, v = np.zeros((1, 5, d), np.float32), np.zeros((1, n, d), np.float32), np.zeros((1, n, d), np.float32)
+    q[:, :, 0] = 1
+    k[0, 1:, 0] = -8 * np.linspace(84.5, 86.5, n - 1)
+    v[0, 1:] = np.abs(O.normal((n - 1, d), 9)) * np.float32(1e30)
+    out = empty((1, 5, d)).fill_(float("nan"))
+    ctx.sdpa(dev(q), dev(k), dev(v), out, E.FP32, 1, 1, 5, n, d, (5 * d, d, n * d, d, n * d, d, 5 * d, d))
+    ref = sdpa_reference(q, k, v)
+    assert np.abs(host(out) - ref).max() <= 2e-5 * np.abs(ref).max()

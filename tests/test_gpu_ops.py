@@ -469,3 +469,20 @@ def test_sdpa_fp32_small_probabilities(ctx):
     ctx.sdpa(dev(q), dev(k), dev(v), out, E.FP32, 1, 1, 5, n, d, (5 * d, d, n * d, d, n * d, d, 5 * d, d))
     ref = sdpa_reference(q, k, v)
     assert np.abs(host(out) - ref).max() <= 2e-5 * np.abs(ref).max()
+
+
+def test_sdpa_fp32_fully_masked_row(ctx):
+    # A query with every key masked out has no result (0 / 0), and does not send the 127
+    # others of its workgroup to the FP32 matrix cores: their bits stay the same.
+    n, d = 130, 128
+    q, k, v = (dev(O.normal((1, n, d), i)) for i in (7, 8, 9))
+    mask = O.normal((n, n), 10)
+    outs = []
+    for _ in range(2):
+        out = empty((1, n, d)).fill_(0)
+        ctx.sdpa(q, k, v, out, E.FP32, 1, 1, n, n, d, (n * d, d) * 4, mask=dev(mask), mask_heads=1, mask_rows=n)
+        outs.append(host(out))
+        mask[5] = -np.inf
+    assert np.all(np.isnan(outs[1][0, 5]))
+    rest = np.delete(np.arange(n), 5)
+    assert np.array_equal(outs[0][0, rest], outs[1][0, rest])

@@ -98,8 +98,10 @@ struct ernie_hip_ctx {
     DeviceBuffer head_ws;  // head intermediates
     DeviceBuffer dit_act;  // run_dit activations: x [S][dim], c, mods
     DeviceBuffer split_ws;   // GEMM tail-row split-K partial sums
-    DeviceBuffer gemm_ws;    // the same for ernie_hip_gemm (from the start; none without memory)
-    bool gemm_ws_null = false;  // last used on the null stream
+    // The same for ernie_hip_gemm: one for calls on the null stream, one for those on other
+    // streams (gemm_workspace).
+    DeviceBuffer gemm_ws[2];
+    bool gemm_ws_tried[2] = {false, false};
     DeviceBuffer rope_pack;  // [S][64] (cos, sin) pairs of the rotary angles, per call
     DeviceBuffer text_ws;    // text block activations
     DeviceBuffer ones;       // FP32 ones: unit gates of the text block's residual epilogues
@@ -981,12 +983,6 @@ int ernie_hip_create(int device, ernie_hip_ctx** out)
     }
     ctx->stream = ctx->own_stream;
     if (scratch_init(device) == 0) ctx->scratch = scratch_address(device);
-    if (hipMalloc(&ctx->gemm_ws.ptr, split_bytes(0, 1)) == hipSuccess) {
-        ctx->gemm_ws.bytes = split_bytes(0, 1);
-    } else {
-        ctx->gemm_ws.ptr = nullptr;
-        (void)hipGetLastError();
-    }
     *out = ctx;
     return ERNIE_OK;
 }
@@ -1006,7 +1002,7 @@ void ernie_hip_destroy(ernie_hip_ctx* ctx)
     dev_free(ctx->head_ws);
     dev_free(ctx->dit_act);
     dev_free(ctx->split_ws);
-    dev_free(ctx->gemm_ws);
+    for (DeviceBuffer& b : ctx->gemm_ws) dev_free(b);
     dev_free(ctx->rope_pack);
     for (hipEvent_t e : ctx->event_pool) (void)hipEventDestroy(e);
     for (hipEvent_t e : ctx->seq_events) (void)hipEventDestroy(e);
@@ -1186,6 +1182,40 @@ int ernie_hip_residual_add(ernie_hip_ctx* ctx, const void* a, int a_dtype, const
     return kernel_status(ctx, residual_add(a, a_dtype, b, b_dtype, out, count, ctx->stream), "residual_add");
 }
 
+// Split-K scratch for an ernie_hip_gemm call, allocated by the first call that can use it.
+// Calls that share a buffer are ordered: on the null stream by the stream, on other streams
+// by set_stream, which waits for the one it leaves (but not for the null stream, whose
+// calls have their own buffer). A call without scratch computes every tile over all of K:
+// a captured call (its graph may be replayed beside other work), one on the per-thread
+// stream (a stream of each calling thread), and every call when the allocation failed
+// (these calls need no memory otherwise).
+static void gemm_workspace(ernie_hip_ctx* ctx, GemmArgs& g)
+{
+    if (ctx->stream == hipStreamPerThread) return;
+    const bool null_stream = !ctx->stream || ctx->stream == hipStreamLegacy;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (!null_stream &&
+        (hipStreamIsCapturing(ctx->stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone))
+        return;
+    DeviceBuffer& b = ctx->gemm_ws[null_stream];
+    if (!ctx->gemm_ws_tried[null_stream]) {
+        ctx->gemm_ws_tried[null_stream] = true;
+        // Relaxed: the allocation is no part of a capture that another stream may have
+        // under way, and must not end it.
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        if (hipMalloc(&b.ptr, split_bytes(0, 1)) == hipSuccess) {
+            b.bytes = split_bytes(0, 1);
+        } else {
+            b.ptr = nullptr;
+            (void)hipGetLastError();
+        }
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+    g.split_ws = b.ptr;
+    g.split_ws_bytes = b.bytes;
+}
+
 int ernie_hip_gemm(ernie_hip_ctx* ctx, const void* a, long lda, const void* w, long ldw, const float* bias, void* c,
                    long ldc, int m, int n, int k, int dtype, int out_dtype)
 {
@@ -1194,19 +1224,7 @@ int ernie_hip_gemm(ernie_hip_ctx* ctx, const void* a, long lda, const void* w, l
     GemmArgs g;
     g.A = a; g.lda = lda; g.W = w; g.ldw = ldw; g.M = m; g.N = n; g.K = k; g.dtype = dtype;
     g.epilogue = EPI_STORE; g.C = c; g.ldc = ldc; g.c_dtype = out_dtype; g.bias = bias;
-    // The context's split-K scratch for these calls, which are ordered on one stream:
-    // set_stream waits for the old one, and a call that leaves the null stream waits for
-    // it here. A captured call takes none (its graph may be replayed beside other work):
-    // every tile then takes all of K.
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    const bool eager = !ctx->stream || (hipStreamIsCapturing(ctx->stream, &capture) == hipSuccess &&
-                                        capture == hipStreamCaptureStatusNone);
-    if (eager && ctx->gemm_ws.ptr && gemm_may_split(g)) {
-        if (ctx->stream && ctx->gemm_ws_null) (void)hipStreamSynchronize(nullptr);
-        ctx->gemm_ws_null = !ctx->stream;
-        g.split_ws = ctx->gemm_ws.ptr;
-        g.split_ws_bytes = ctx->gemm_ws.bytes;
-    }
+    if (gemm_may_split(g)) gemm_workspace(ctx, g);
     return kernel_status(ctx, gemm(g, ctx->stream), "gemm");
 }
 

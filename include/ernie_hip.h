@@ -89,7 +89,11 @@ int ernie_hip_residual_add(ernie_hip_ctx* ctx, const void* a, int a_dtype, const
  * (block.ncnn.param line 19 etc.): C[m][n] = sum_k A[m][k] W[n][k] (+ bias[n]).
  * A, W row strides lda / ldw (elements, multiples of 8 for 16-bit, 4 for FP32;
  * 16-byte aligned bases); K % 32 == 0 (16-bit) or K % 16 == 0 (FP32).
- * out_dtype: FP32 or equal to dtype. */
+ * out_dtype: FP32 or equal to dtype.
+ * The first call that can use it allocates 128 MiB of split-K scratch, kept with the context
+ * (one for the null stream, one for other streams; none without memory). Captured calls
+ * and calls on hipStreamPerThread take none, so that they may add the same products in
+ * another order than an eager call does. */
 int ernie_hip_gemm(ernie_hip_ctx* ctx, const void* a, long lda, const void* w, long ldw, const float* bias,
                    void* c, long ldc, int m, int n, int k, int dtype, int out_dtype);
 /* "SDPA" with 5=1 (attn mask) -> ErnieSDPA::forward (src/ernie_attention.cpp:201-230):

@@ -213,6 +213,44 @@ def test_gemm_tail_rows_below_few_tiles(ctx, dt, m, n, k):
     assert g["passed"], g
 
 
+def test_gemm_scratch_is_allocated_when_used():
+    # A context takes no scratch until a matrix product of its own can use it.
+    import torch
+    before = torch.cuda.mem_get_info()[0]
+    c = E.Context(0)
+    assert before - torch.cuda.mem_get_info()[0] < 64 << 20
+    c.close()
+
+
+def test_gemm_scratch_beside_a_capture(ctx):
+    # Calls on the null stream, then on another one while a third stream is captured in the
+    # strictest mode: the capture stays valid, and both calls have their results.
+    import torch
+    m, n, k = 300, 256, 4096
+    a, w = O.normal((m, k), 3), O.normal((n, k), 4, std=0.02)
+    ref = O.gemm_nt(stored(a, E.FP16), stored(w, E.FP16)).astype(np.float64)
+    ad, wd, outs = dev(a, E.FP16), dev(w, E.FP16), [empty((m, n)).fill_(float("nan")) for _ in range(2)]
+    side, captured, graph = torch.cuda.Stream(), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    x = empty((4096,)).fill_(0)
+    torch.cuda.synchronize()
+    try:
+        ctx.call("set_stream", None)
+        ctx.gemm(ad, k, wd, k, outs[0], n, m, n, k, E.FP16, E.FP32)
+        ctx.call("set_stream", E.c_vp(side.cuda_stream))
+        with torch.cuda.graph(graph, stream=captured, capture_error_mode="global"):
+            x.add_(1)
+            ctx.gemm(ad, k, wd, k, outs[1], n, m, n, k, E.FP16, E.FP32)
+    finally:
+        ctx.call("set_stream", E.c_vp(torch.cuda.current_stream().cuda_stream))
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+    assert np.all(host(x) == 3)
+    for out in outs:
+        g = kat.gate(host(out), ref, 0, 1e-5, 1e-5)
+        assert g["passed"], g
+
+
 def test_gemm_rejects_unsupported_shapes(ctx):
     a, c = empty((4, 40), E.FP16), empty((4, 8))
     with pytest.raises(E.ErnieError):

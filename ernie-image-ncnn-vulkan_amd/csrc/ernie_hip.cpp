@@ -1224,6 +1224,7 @@ int ernie_hip_gemm(ernie_hip_ctx* ctx, const void* a, long lda, const void* w, l
     GemmArgs g;
     g.A = a; g.lda = lda; g.W = w; g.ldw = ldw; g.M = m; g.N = n; g.K = k; g.dtype = dtype;
     g.epilogue = EPI_STORE; g.C = c; g.ldc = ldc; g.c_dtype = out_dtype; g.bias = bias;
+    g.alone = true;
     if (gemm_may_split(g)) gemm_workspace(ctx, g);
     return kernel_status(ctx, gemm(g, ctx->stream), "gemm");
 }

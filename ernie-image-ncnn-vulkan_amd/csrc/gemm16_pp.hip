@@ -1093,6 +1093,28 @@ static bool light_assign(pingpong::Params& p, int grid)
     return ok;
 }
 
+// The time of a K step in a tile of 64 n rows, to that of a full tile.
+constexpr double kTileSteps[5] = {0, 0.62, 0.74, 0.85, 1.0};
+
+// Whether cutting tiles into sp K parts pays in a call of its own (ernie_hip_gemm; the
+// blocks' plans were chosen on the blocks' own times). A K step of a full tile takes
+// 0.53 us while at most 128 workgroups run and up to 0.72 with all 256 (the chip is
+// power-limited); summing the parts takes 3 us and 0.225 us per MB of them. `tiles` of
+// `height` steps become `items` of `item_height`, with part_rows rows of partial sums in
+// all; `margin` is what the split's side is multiplied by, for what the estimate leaves
+// out. Over 1236 sizes (17 to 4160 rows, 256 to 24576 columns, K 256 to 4096), each
+// measured with and without the split, the choice is within 0.3 % of the faster side on
+// average, and slower than no split by more than 3 % at three sizes (at most 8 %);
+// always splitting was up to 1.8 times slower (320 x 16384 x 1024: 30 us against 55).
+static bool alone_split_pays(int nk, int sp, double height, int tiles, double item_height, int items, int part_rows,
+                             double margin)
+{
+    if (sp < 2) return false;
+    auto step = [](int n) { return 0.53 + 0.0015 * std::max(0, std::min(n, 256) - 128); };
+    const double mb = (double)part_rows * pingpong::BN * sizeof(float) * 1e-6;
+    return margin * (step(items) * item_height * ((nk + sp - 1) / sp) + 3 + 0.225 * mb) < step(tiles) * height * nk;
+}
+
 int gemm16_pingpong(const GemmArgs& a, hipStream_t s)
 {
     // No other kernel takes K-tiled operands or fuses the Q/K epilogue: shapes this one
@@ -1180,7 +1202,12 @@ int gemm16_pingpong(const GemmArgs& a, hipStream_t s)
         // Whole rounds, or one or two rounds at least three quarters full: those run on
         // `even` workgroups with one or two tiles each (a tile takes less time while some
         // CUs idle: the chip is power-limited).
-        const bool near_whole = full % cu_count() == 0 || (rounds <= 2 && 4 * full >= 3 * rounds * cu_count());
+        // A call of its own, whose tail would not be split, needs them only where the tail's
+        // tiles would begin another round: else they run on idle CUs (1056 x 12288 x 4096
+        // 104 us against 114; 1300 x 12288 x 4096, where they do, 171 against 124).
+        const bool near_whole = full % cu_count() == 0 ||
+                                (rounds <= 2 && 4 * full >= 3 * rounds * cu_count() &&
+                                 (!a.alone || full + p.n_tiles > rounds * cu_count()));
         if ((qk || epi_glu(a.epilogue) || a.epilogue == EPI_STORE) && tail_rows > 0 && tail_rows <= 64 &&
             full > 0 && near_whole && p.m_full >= chunks) {
             p.light = 1;
@@ -1206,20 +1233,32 @@ int gemm16_pingpong(const GemmArgs& a, hipStream_t s)
     }
     // A split into sp parts takes at least 16 K steps off a tile: a step of a lone tile is
     // about 0.45 us, the reduction launch 5 to 7 us.
-    auto worth = [&](int sp) { const int nk = a.K / pingpong::BK; return sp > 1 && nk - (nk + sp - 1) / sp >= 16; };
+    const int nk = a.K / pingpong::BK;
+    auto worth = [&](int sp) { return sp > 1 && nk - (nk + sp - 1) / sp >= 16; };
+    // K parts of every one of `tiles` tiles of `rows` rows: enough to cover the CUs once, at
+    // least 4 K steps each, within the scratch.
+    auto parts_of_all = [&](int tiles, int rows) {
+        const size_t per_part = (size_t)tiles * rows * pingpong::BN * sizeof(float);
+        int sp = std::min(kMaxSplit, kSplitTargetItems / tiles);
+        sp = std::min(sp, std::max(1, nk / 4));
+        while (sp > 1 && sp * per_part > a.split_ws_bytes) --sp;
+        return sp;
+    };
     // Too few tiles for the CUs (a short sequence's narrow projections): split every tile
-    // along K, at least 4 K steps per part. A tail of at most 64 rows below one or two
-    // rows of tiles goes into the last of them, as 320-row tiles: half or two thirds of the
-    // tiles, each reading its W once, so that more parts fit the CUs.
-    const bool tall = tail_rows > 0 && tail_rows <= 64 && (p.m_full == 1 || p.m_full == 2);
+    // along K. A tail of at most 64 rows below one or two rows of tiles goes into the last
+    // of them, as 320-row tiles: half or two thirds of the tiles, each reading its W once,
+    // so that more parts fit the CUs.
+    const int flat_tiles = (p.m_full + (p.tail_sub ? 1 : 0)) * p.n_tiles;
+    bool tall = tail_rows > 0 && tail_rows <= 64 && (p.m_full == 1 || p.m_full == 2);
+    if (a.alone && tall && full <= kSplitTargetItems / 2) {
+        const int sp = parts_of_all(full, pingpong::BM + 64);
+        tall = alone_split_pays(nk, sp, 1.0, flat_tiles, 1.25, full * sp, full * sp * (pingpong::BM + 64), 1.2);
+    }
     const int m_tiles = p.m_full + (p.tail_sub && !tall ? 1 : 0);
     p.part_rows = tall ? pingpong::BM + 64 : pingpong::BM;
     if (!p.light && (!p.heavy || tall) && a.split_ws && p.m_full && m_tiles * p.n_tiles <= kSplitTargetItems / 2) {
-        const size_t per_part = (size_t)m_tiles * p.n_tiles * p.part_rows * pingpong::BN * sizeof(float);
-        int sp = std::min(kMaxSplit, kSplitTargetItems / (m_tiles * p.n_tiles));
-        sp = std::min(sp, std::max(1, a.K / pingpong::BK / 4));
-        while (sp > 1 && (size_t)sp * per_part > a.split_ws_bytes) --sp;
-        if (worth(sp)) {
+        const int sp = parts_of_all(m_tiles * p.n_tiles, p.part_rows), items = m_tiles * p.n_tiles * sp;
+        if (worth(sp) && (!a.alone || tall || alone_split_pays(nk, sp, 1.0, flat_tiles, 1.0, items, items * pingpong::BM, 0.95))) {
             p.split = sp;
             p.split_all = 1;
             p.heavy = tall;
@@ -1239,12 +1278,31 @@ int gemm16_pingpong(const GemmArgs& a, hipStream_t s)
         p.split = p.m_full;
         p.part = static_cast<float*>(a.split_ws);
     }
+    // A last round of at most half the CUs: its tiles may be split too (below). A call of its
+    // own does that where it saves enough K steps to pay for up to 84 MB of sums: 768 x 24576 x
+    // 4096 222 -> 171 us, x 2048 127 -> 105, but x 1024 78 -> 76; with a tail, where
+    // both are few, 2368 x 8192 x 4096 197 -> 173, but 780 x 24576 x 4096 200 -> 217.
+    const int last_round = full % kSplitTargetItems;
+    bool late = full > kSplitTargetItems && last_round > 0 && last_round <= kSplitTargetItems / 2;
+    if (late && a.alone) {
+        const int sp = std::min(std::min(kMaxSplit, kSplitTargetItems / last_round), std::max(1, nk / 4));
+        const int saved = nk - (nk + sp - 1) / sp;
+        late = p.tail_sub ? saved >= 96 && last_round <= 64 && p.n_tiles <= 48 : saved >= 48;
+    }
     if (!p.heavy && !p.ride && !p.light && !p.split_all && p.tail_sub && a.split_ws) {
         const size_t per_part = (size_t)p.n_tiles * 64 * p.tail_sub * pingpong::BN * sizeof(float);
         int sp = std::min(kMaxSplit, std::max(1, kSplitTargetItems / p.n_tiles));
-        sp = std::min(sp, std::max(1, a.K / pingpong::BK / 4));
+        sp = std::min(sp, std::max(1, nk / 4));
         while (sp > 1 && (size_t)sp * per_part > a.split_ws_bytes) --sp;
-        p.split = worth(sp) ? sp : 1;
+        bool split = worth(sp);
+        if (split && a.alone) {
+            const double h = kTileSteps[p.tail_sub];
+            const int items = p.n_tiles * sp;
+            if (!full) split = alone_split_pays(nk, sp, h, flat_tiles, h, items, items * 64 * p.tail_sub, 0.85);
+            else if (full % kSplitTargetItems == 0) split = alone_split_pays(nk, sp, h, kSplitTargetItems, h, kSplitTargetItems, items * 64 * p.tail_sub, 1.3);
+            else split = late;
+        }
+        p.split = split ? sp : 1;
         p.part = static_cast<float*>(a.split_ws);
     }
     // A last round of workgroups at most half full (the full tiles modulo one per
@@ -1253,10 +1311,8 @@ int gemm16_pingpong(const GemmArgs& a, hipStream_t s)
     p.late = 0;
     p.late_split = 1;
     p.late_part = nullptr;
-    const int last_round = full % kSplitTargetItems;
     // (Not for the fused Q/K epilogue, whose rows are finished per tile.)
-    if (!qk && !p.heavy && !p.ride && !p.light && !p.split_all && a.split_ws && full > kSplitTargetItems &&
-        last_round <= kSplitTargetItems / 2 && last_round > 0) {
+    if (!qk && !p.heavy && !p.ride && !p.light && !p.split_all && a.split_ws && late) {
         const size_t tail_bytes =
             p.tail_sub ? ((size_t)p.split * p.n_tiles * 64 * p.tail_sub * pingpong::BN * sizeof(float) + 255) / 256 * 256 : 0;
         const size_t per_part = (size_t)last_round * pingpong::BM * pingpong::BN * sizeof(float);

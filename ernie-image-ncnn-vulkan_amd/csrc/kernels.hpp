@@ -55,6 +55,9 @@ struct GemmArgs {
     // share it; calls that run concurrently must not.
     void* split_ws = nullptr;
     size_t split_ws_bytes = 0;
+    // A call of its own (ernie_hip_gemm) rather than a block's or head's product: 16-bit
+    // products are then split only where that was measured to pay over all sizes.
+    bool alone = false;
     // EPI_QKROPE: Q / K columns [0, qk_cols) (K heads from k_col), their gammas [128],
     // and each row's rotary angles as rope_pack writes them, [M][64] (cos, sin) pairs.
     int qk_cols = 0;

@@ -251,6 +251,41 @@ def test_gemm_scratch_beside_a_capture(ctx):
         assert g["passed"], g
 
 
+def captured_gemm(ctx, *args):
+    """The call recorded into a graph, which takes no scratch, and replayed."""
+    import torch
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    try:
+        ctx.call("set_stream", E.c_vp(stream.cuda_stream))
+        with torch.cuda.graph(graph, stream=stream, capture_error_mode="relaxed"):
+            ctx.gemm(*args)
+    finally:
+        ctx.call("set_stream", E.c_vp(torch.cuda.current_stream().cuda_stream))
+    graph.replay()
+    torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("m,n,k,split", [(320, 16384, 1024, False), (2090, 4096, 1024, False), (400, 24576, 1024, False),
+                                         (1152, 8192, 1024, False), (1568, 12288, 1024, False), (1056, 12288, 1024, False),
+                                         (100, 1024, 4096, True), (320, 1024, 4096, True), (512, 1024, 4096, True),
+                                         (2368, 8192, 4096, True), (1152, 16384, 4096, True)])
+def test_gemm_split_where_it_pays(ctx, m, n, k, split):
+    # Enough tiles or few K steps: no split (nor light tiles), so the bits of a captured call,
+    # which has no scratch to split with. Few tiles and many K steps: parts of K summed
+    # in another order. Both against the products of the stored values.
+    import torch
+    a, w = dev(O.normal((m, k), 3), E.FP16), dev(O.normal((n, k), 4, std=0.02), E.FP16)
+    c, whole = empty((m, n)).fill_(float("nan")), empty((m, n)).fill_(float("nan"))
+    ctx.gemm(a, k, w, k, c, n, m, n, k, E.FP16, E.FP32)
+    captured_gemm(ctx, a, k, w, k, whole, n, m, n, k, E.FP16, E.FP32)
+    assert torch.equal(c, whole) == (not split)
+    ref = a.double() @ w.double().T
+    for x in (c, whole):
+        # k FP32 roundings of sums that grow to the result: sqrt(k) 2^-24 of it at most.
+        assert float((x - ref).norm() / ref.norm()) < math.sqrt(k) * 2**-24
+
+
 def test_gemm_rejects_unsupported_shapes(ctx):
     a, c = empty((4, 40), E.FP16), empty((4, 8))
     with pytest.raises(E.ErnieError):

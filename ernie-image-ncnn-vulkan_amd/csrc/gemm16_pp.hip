@@ -1093,6 +1093,13 @@ static bool light_assign(pingpong::Params& p, int grid)
     return ok;
 }
 
+// Whether the few-row kernel ends before one round of unsplit tiles (times in us).
+static bool skinny_pays(int M, int N, int K)
+{
+    const double groups = skinny_workgroups(N), w = (double)N * K * 2, a = groups * M * K * 2;
+    return 5 + w / 6e6 + a / 13e6 < 4 + 0.36 * (K / pingpong::BK);
+}
+
 // The time of a K step in a tile of 64 n rows, to that of a full tile.
 constexpr double kTileSteps[5] = {0, 0.62, 0.74, 0.85, 1.0};
 
@@ -1158,9 +1165,16 @@ int gemm16_pingpong(const GemmArgs& a, hipStream_t s)
     }
     // At most 16 rows: 16 x 4096 x 4096 12 us against 17 split along K here, 16 x 9216 x
     // 3072 21 against 22; from 24 rows on the split is faster (19 against 21 us at 6144 x
-    // 3072), since every workgroup of the few-row kernel reads all of A. Without split
-    // scratch (a captured call) up to 128 rows: 128 x 3072 x 9216 91 us against 196.
-    if (a.M <= (a.split_ws ? 16 : kSkinnyRows)) return gemm16_skinny(a, p.vec, s);
+    // 3072), since every workgroup of the few-row kernel reads all of A. A plain product
+    // without split scratch (a captured call) takes it up to 128 rows where the reads of W
+    // (at 6 TB/s) and A (13 TB/s, mostly from L2) end before one round of tiles over all of
+    // K: 128 x 3072 x 9216 79 us against 158, but 128 x 65536 x 3072 276 against 102. Over 260
+    // captured sizes (128 to 65536 columns, K 512 to 9216) the choice is within 1.2 % of
+    // the faster one on average. A call of its own has no more than 16 rows there either:
+    // 16 x 65536 x 512 26 us against 18.
+    const bool few = a.M <= 16 && !a.alone;
+    if (few || (!a.split_ws && a.M <= kSkinnyRows && a.epilogue == EPI_STORE && skinny_pays(a.M, a.N, a.K)))
+        return gemm16_skinny(a, p.vec, s);
     p.qk_cols = a.qk_cols; p.k_col = a.k_col; p.gq = a.gq; p.gk = a.gk; p.cs_t = a.cs_t;
     p.qk_eps = a.qk_eps;
     p.w_bytes = (uint32_t)((long)a.N * a.ldw * 2);

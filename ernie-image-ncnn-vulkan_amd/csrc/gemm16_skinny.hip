@@ -175,11 +175,10 @@ void launch_mb(const Params& p, hipStream_t s)
     const dim3 block(64 * WAVES);
     if constexpr (epi_glu(EPI)) {
         hipLaunchKernelGGL((kernel<T, OutT, EPI, MB, 2, U>), dim3(p.N / 32), block, 0, s, p);
-    } else if (p.N <= 16 * 512) {
-        // 16 columns per workgroup while that is at most two workgroups per CU.
-        hipLaunchKernelGGL((kernel<T, OutT, EPI, MB, 1, U>), dim3((p.N + 15) / 16), block, 0, s, p);
+    } else if (p.N <= kSkinnyNarrow) {
+        hipLaunchKernelGGL((kernel<T, OutT, EPI, MB, 1, U>), dim3(skinny_workgroups(p.N)), block, 0, s, p);
     } else {
-        hipLaunchKernelGGL((kernel<T, OutT, EPI, MB, 2, U>), dim3((p.N + 31) / 32), block, 0, s, p);
+        hipLaunchKernelGGL((kernel<T, OutT, EPI, MB, 2, U>), dim3(skinny_workgroups(p.N)), block, 0, s, p);
     }
 }
 

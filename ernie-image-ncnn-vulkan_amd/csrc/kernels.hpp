@@ -77,6 +77,10 @@ int gemm16_pingpong(const GemmArgs& a, hipStream_t stream);
 // gemm16_pingpong with arguments it has checked. vec: every output row, residual row and
 // vector is aligned for four columns at a time.
 constexpr int kSkinnyRows = 128;
+// Its workgroups for N columns of a plain product: 16 columns each while that is at most two
+// per CU, else 32.
+constexpr int kSkinnyNarrow = 16 * 512;
+inline int skinny_workgroups(int N) { return N <= kSkinnyNarrow ? (N + 15) / 16 : (N + 31) / 32; }
 int gemm16_skinny(const GemmArgs& a, bool vec, hipStream_t stream);
 
 // ---- flash SDPA ---------------------------------------------------------------

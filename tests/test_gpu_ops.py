@@ -286,6 +286,25 @@ def test_gemm_split_where_it_pays(ctx, m, n, k, split):
         assert float((x - ref).norm() / ref.norm()) < math.sqrt(k) * 2**-24
 
 
+@pytest.mark.parametrize("m,n,k,few", [(100, 32768, 512, False), (64, 32768, 512, False), (16, 65536, 512, False),
+                                       (128, 3072, 3072, True), (40, 8224, 1024, True), (100, 8224, 3072, True)])
+def test_gemm_few_rows_where_they_pay(ctx, m, n, k, few):
+    # A captured call of few rows: past the columns where every workgroup's reading of A costs
+    # more than tiles over all of K, the bits of the first rows of a call with more rows
+    # (whole tiles); below, the few-row kernel's, which adds its waves' parts of K.
+    import torch
+    rows = 260
+    a, w = dev(O.normal((rows, k), 3), E.BF16), dev(O.normal((n, k), 4, std=0.02), E.BF16)
+    c, more = empty((m, n)).fill_(float("nan")), empty((rows, n)).fill_(float("nan"))
+    captured_gemm(ctx, a, k, w, k, c, n, m, n, k, E.BF16, E.FP32)
+    captured_gemm(ctx, a, k, w, k, more, n, rows, n, k, E.BF16, E.FP32)
+    assert torch.equal(c, more[:m]) == (not few)
+    ref = a.double() @ w.double().T
+    for x in (c, more):
+        # k FP32 roundings of sums that grow to the result: sqrt(k) 2^-24 of it at most.
+        assert float((x - ref[:len(x)]).norm() / ref[:len(x)].norm()) < math.sqrt(k) * 2**-24
+
+
 def test_gemm_rejects_unsupported_shapes(ctx):
     a, c = empty((4, 40), E.FP16), empty((4, 8))
     with pytest.raises(E.ErnieError):

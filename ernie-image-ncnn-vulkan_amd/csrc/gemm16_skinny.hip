@@ -1,13 +1,15 @@
 // SPDX-License-Identifier: MIT
-// 16-bit GEMM for few rows (a short prompt's or a thumbnail's projections), C[M,N] =
-// A[M,K] * W[N,K]^T with FP32 accumulation and the epilogues of gemm16_pp.hip.
+// 16-bit GEMM for few rows, C[M,N] = A[M,K] * W[N,K]^T with FP32 accumulation and the
+// epilogues of gemm16_pp.hip: products of at most 16 rows, and plain ones without split
+// scratch of up to 128 rows and not too many columns (gemm16_pingpong decides).
 //
-// With at most 128 rows the product is bound by reading W once. The 256 x 256 tiles of
-// the general kernel stage it through LDS for mostly empty rows and need a split along
-// K, with a reduction launch, to fill the chip. Here a workgroup owns 16 or 32 columns
-// and all rows; its 8 waves cut K between them, each reading its operands straight into
-// MFMA fragments (no LDS, no barrier in the loop, two groups of K steps in flight), and
-// their sums are added through LDS in wave order, so that one launch stores the result.
+// With at most 16 rows the product is bound by reading W once. The 256 x 256 tiles of the
+// general kernel stage it through LDS for mostly empty rows and need a split along K, with
+// a reduction launch, to fill the chip. Here a workgroup owns 16 or 32 columns and all
+// rows; its 8 waves cut K between them, each reading its operands straight into MFMA
+// fragments (no LDS, no barrier in the loop, two groups of K steps in flight), and their
+// sums are added through LDS in wave order, so that one launch stores the result. Every
+// workgroup reads all of A, which is what bounds it with more rows and many columns.
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -182,23 +184,31 @@ void launch_mb(const Params& p, hipStream_t s)
     }
 }
 
+// More than 16 rows: plain products only. Returns -1 for others.
 template <typename T, typename OutT, int EPI>
-void launch(const Params& p, hipStream_t s)
+int launch(const Params& p, hipStream_t s)
 {
-    if (p.M <= 16) launch_mb<T, OutT, EPI, 1>(p, s);
-    else if (p.M <= 32) launch_mb<T, OutT, EPI, 2>(p, s);
-    else if (p.M <= 64) launch_mb<T, OutT, EPI, 4>(p, s);
-    else launch_mb<T, OutT, EPI, 8>(p, s);
+    if (p.M <= 16) {
+        launch_mb<T, OutT, EPI, 1>(p, s);
+        return 0;
+    }
+    if constexpr (EPI == EPI_STORE) {
+        if (p.M <= 32) launch_mb<T, OutT, EPI, 2>(p, s);
+        else if (p.M <= 64) launch_mb<T, OutT, EPI, 4>(p, s);
+        else launch_mb<T, OutT, EPI, 8>(p, s);
+        return 0;
+    }
+    return -1;
 }
 
 template <typename T>
-void launch_dtype(const GemmArgs& a, const Params& p, hipStream_t s)
+int launch_dtype(const GemmArgs& a, const Params& p, hipStream_t s)
 {
-    if (a.epilogue == EPI_GATE_RESID) launch<T, float, EPI_GATE_RESID>(p, s);
-    else if (a.epilogue == EPI_SWIGLU) launch<T, T, EPI_SWIGLU>(p, s);
-    else if (a.epilogue == EPI_GEGLU) launch<T, T, EPI_GEGLU>(p, s);
-    else if (a.c_dtype == DT_F32) launch<T, float, EPI_STORE>(p, s);
-    else launch<T, T, EPI_STORE>(p, s);
+    if (a.epilogue == EPI_GATE_RESID) return launch<T, float, EPI_GATE_RESID>(p, s);
+    if (a.epilogue == EPI_SWIGLU) return launch<T, T, EPI_SWIGLU>(p, s);
+    if (a.epilogue == EPI_GEGLU) return launch<T, T, EPI_GEGLU>(p, s);
+    if (a.c_dtype == DT_F32) return launch<T, float, EPI_STORE>(p, s);
+    return launch<T, T, EPI_STORE>(p, s);
 }
 
 }  // namespace skinny
@@ -216,12 +226,12 @@ int gemm16_skinny(const GemmArgs& a, bool vec, hipStream_t s)
     p.c_ss = a.c_k32_rows ? 32L * a.c_k32_rows : 32;
     p.bias = a.bias; p.resid = a.resid; p.ld_resid = a.ld_resid; p.gate = a.gate;
     p.vec = vec;
-    if (a.dtype == DT_F16) skinny::launch_dtype<f16>(a, p, s);
-    else skinny::launch_dtype<bf16>(a, p, s);
+    int rc = a.dtype == DT_F16 ? skinny::launch_dtype<f16>(a, p, s) : skinny::launch_dtype<bf16>(a, p, s);
+    if (rc) return rc;
     if (a.epilogue == EPI_QKROPE) {
         // Q and K columns were stored permuted and rounded: normalised, rotated and put in
         // natural order as for the split rows of the general kernel.
-        const int rc = qk_norm_rope_permuted(a.C, a.dtype, 0, a.M, (int)(a.k_col / 128), (int)((a.qk_cols - a.k_col) / 128),
+        rc = qk_norm_rope_permuted(a.C, a.dtype, 0, a.M, (int)(a.k_col / 128), (int)((a.qk_cols - a.k_col) / 128),
                                              a.ldc, a.k_col, a.gq, a.gk, a.cs_t, a.qk_eps, s);
         if (rc) return rc;
     }

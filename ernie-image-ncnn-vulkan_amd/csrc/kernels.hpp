@@ -73,8 +73,8 @@ bool gemm_may_split(const GemmArgs& a);
 // The ping-pong 16-bit kernel (gemm16_pp.hip); returns 1 without launching when
 // the shape needs the register-staged kernel instead (operands of 2 GiB or more).
 int gemm16_pingpong(const GemmArgs& a, hipStream_t stream);
-// The 16-bit kernel for at most kSkinnyRows rows (gemm16_skinny.hip), called by
-// gemm16_pingpong with arguments it has checked. vec: every output row, residual row and
+// The 16-bit kernel for at most 16 rows, or kSkinnyRows of a plain product
+// (gemm16_skinny.hip), called by gemm16_pingpong with arguments it has checked. vec: every output row, residual row and
 // vector is aligned for four columns at a time.
 constexpr int kSkinnyRows = 128;
 // Its workgroups for N columns of a plain product: 16 columns each while that is at most two

@@ -287,7 +287,8 @@ def test_gemm_split_where_it_pays(ctx, m, n, k, split):
 
 
 @pytest.mark.parametrize("m,n,k,few", [(100, 32768, 512, False), (64, 32768, 512, False), (16, 65536, 512, False),
-                                       (128, 3072, 3072, True), (40, 8224, 1024, True), (100, 8224, 3072, True)])
+                                       (32, 3072, 3072, True), (128, 3072, 3072, True), (40, 8224, 1024, True),
+                                       (100, 8224, 3072, True)])
 def test_gemm_few_rows_where_they_pay(ctx, m, n, k, few):
     # A captured call of few rows: past the columns where every workgroup's reading of A costs
     # more than tiles over all of K, the bits of the first rows of a call with more rows

@@ -1259,12 +1259,15 @@ int gemm16_pingpong(const GemmArgs& a, hipStream_t s)
         return sp;
     };
     // Too few tiles for the CUs (a short sequence's narrow projections): split every tile
-    // along K. A tail of at most 64 rows below one or two rows of tiles goes into the last
-    // of them, as 320-row tiles: half or two thirds of the tiles, each reading its W once,
-    // so that more parts fit the CUs.
+    // along K. Where a tail of at most 64 rows below one or two rows of tiles makes them too
+    // many for that, it goes into the last of them, as 320-row tiles (288 x 24576 x 4096 in a
+    // block: 122 us with a split tail row, 84 so). Where 256-row tiles can all be split, 320-row
+    // ones are no faster: blocks of 260 to 576 tokens measured 1 % (width 4096) to 9 % (1024)
+    // slower with them at one row of tiles, -4 % (3072) to 6 % (2048) at two.
     const int flat_tiles = (p.m_full + (p.tail_sub ? 1 : 0)) * p.n_tiles;
-    bool tall = tail_rows > 0 && tail_rows <= 64 && (p.m_full == 1 || p.m_full == 2);
-    if (a.alone && tall && full <= kSplitTargetItems / 2) {
+    bool tall = tail_rows > 0 && tail_rows <= 64 && (p.m_full == 1 || p.m_full == 2) &&
+                flat_tiles > kSplitTargetItems / 2 && full <= kSplitTargetItems / 2;
+    if (tall && a.alone) {
         const int sp = parts_of_all(full, pingpong::BM + 64);
         tall = alone_split_pays(nk, sp, 1.0, flat_tiles, 1.25, full * sp, full * sp * (pingpong::BM + 64), 1.2);
     }

@@ -72,6 +72,23 @@ def test_block_last_round_split_against_oracle(ctx, dt):
 
 
 @pytest.mark.parametrize("dt", [E.FP16, E.BF16], ids=lambda d: NAMES[d])
+@pytest.mark.parametrize("S,image", [(257, (16, 15)), (320, (16, 18))])
+def test_block_tall_split_tiles_against_oracle(ctx, dt, S, image):
+    # Width 1024, FFN 8448, one full row of tiles and a tail of 1 and 64 rows: the up/gate
+    # GEMM's 66 tiles are 320 rows tall and split along K, and its reduction writes the
+    # K-tiled GEGLU output. The narrower projections split 256-row tiles: 24 of Q/K/V, whose
+    # rows are all normalised and rotated after the sums, 8 of the gated residuals.
+    dim, ffn = 1024, 8448
+    w = small_block(dim=dim, ffn=ffn, seed=17)
+    x, mods, cos, sin, mask = small_inputs(S=S, dim=dim, image=image, valid=9, seed=18)
+    ctx.block_upload(5, w, dim, ffn, dt)
+    got = run_block(ctx, 5, x, mods, cos, sin, mask, int(np.sum(mask == 0)))
+    g = kat.gate(got, O.block_forward(w, x, mods, cos, sin, mask), *kat.BLOCK_GATES[NAMES[dt]])
+    assert g["passed"], g
+    ctx.call("block_release", 5)
+
+
+@pytest.mark.parametrize("dt", [E.FP16, E.BF16], ids=lambda d: NAMES[d])
 def test_block_heavy_tail_tiles_against_oracle(ctx, dt):
     # Width 1024 (8 heads), FFN 4096, S = 5160 = 20 x 256 + 40 (64 x 80 image tokens,
     # 40 text slots, 30 valid). The up/gate GEMM has 20 x 32 = 640 full tiles, two and a

@@ -125,6 +125,21 @@ def test_text_block_ragged_tiles_against_oracle(ctx, dt):
 
 
 @pytest.mark.parametrize("dt", [E.FP16, E.BF16], ids=lambda d: NAMES[d])
+def test_text_block_split_tiles_against_oracle(ctx, dt):
+    # Width 1024, FFN 8448, 300 tokens: the gate/up GEMM's 66 tiles are 320 rows tall and split
+    # along K, with the SwiGLU in the reduction; the other products split 256-row tiles.
+    hidden, heads, kv, ffn, S = 1024, 8, 2, 8448, 300
+    w = small_text_block(seed=48, hidden=hidden, heads=heads, kv_heads=kv, ffn=ffn)
+    ctx.text_block_upload(4, w, hidden, heads, kv, ffn, dt)
+    cos, sin, mask = O.text_constants(yarn_like_frequencies(), S)
+    x = O.normal((S, hidden), 49, std=0.2)
+    ref = O.text_block_forward(w, x, cos, sin, mask, heads, kv)
+    g = kat.gate(run_text_block(ctx, 4, x, cos, sin, None, causal=True), ref, *kat.TEXT_GATES[NAMES[dt]])
+    assert g["passed"], g
+    ctx.call("text_block_release", 4)
+
+
+@pytest.mark.parametrize("dt", [E.FP16, E.BF16], ids=lambda d: NAMES[d])
 @pytest.mark.parametrize("S", [1, 16])
 def test_text_block_few_tokens_against_oracle(ctx, dt, S):
     # The GEMMs' few-row kernel with the SwiGLU and residual epilogues.

@@ -94,7 +94,8 @@ def test_block_heavy_tail_tiles_against_oracle(ctx, dt):
     # 40 text slots, 30 valid). The up/gate GEMM has 20 x 32 = 640 full tiles, two and a
     # half rounds of 256 workgroups, so its last row of tiles takes the 40 tail rows as
     # 320-row tiles (rows past S are computed and not stored) instead of a split tail
-    # row; the other GEMMs have too few tiles for that and keep their split tails.
+    # row. The Q/K/V GEMM's 240 full tiles, one partial round, take them as light tiles;
+    # the output and down projections' 80 full tiles split every tile along K.
     dim, ffn = 1024, 4096
     w = small_block(dim=dim, ffn=ffn, seed=11)
     x, mods, cos, sin, mask = small_inputs(S=5160, dim=dim, image=(64, 80), valid=30, seed=12)
@@ -127,6 +128,25 @@ def test_block_light_tail_tiles_against_oracle(ctx, dt, ffn):
     g = kat.gate(got, ref, *kat.BLOCK_GATES[NAMES[dt]])
     assert g["passed"], g
     np.testing.assert_array_equal(run_block(ctx, 7, x, mods, cos, sin, mask, valid), got)  # repeat-deterministic
+    ctx.call("block_release", 7)
+
+
+@pytest.mark.parametrize("dt", [E.FP16, E.BF16], ids=lambda d: NAMES[d])
+def test_block_light_tail_tiles_on_partial_rounds(ctx, dt):
+    # Width 2048, FFN 6144, S = 8 x 256 + 50: 192 full tiles in the Q/K/V GEMM and 384 in
+    # up/gate, three quarters of one and of two rounds; the 50 tail rows go as four 16-row
+    # chunks into some of them, with the Q/K norm and rotary and the GEGLU of each chunk.
+    dim, ffn, S = 2048, 6144, 2098
+    w = small_block(dim=dim, ffn=ffn, seed=19)
+    x, mods, cos, sin, mask = small_inputs(S=S, dim=dim, image=(32, 64), valid=30, seed=20)
+    ctx.block_upload(7, w, dim, ffn, dt)
+    got = run_block(ctx, 7, x, mods, cos, sin, mask, int(np.sum(mask == 0)))
+    ref = O.block_forward(w, x, mods, cos, sin, mask)
+    g = kat.gate(got, ref, *kat.BLOCK_GATES[NAMES[dt]])
+    assert g["passed"], g
+    # The tail rows by themselves: a misplaced chunk is a few rows of 2098.
+    g = kat.gate(got[2048:], ref[2048:], *kat.BLOCK_GATES[NAMES[dt]])
+    assert g["passed"], g
     ctx.call("block_release", 7)
 
 
@@ -373,21 +393,23 @@ def test_facade_block_sequence_validation_and_parity():
     fac.close()
 
 
-@pytest.mark.parametrize("dim,ffn,S,image,valid", [(4096, 1024, 4160, (64, 64), 40), (1024, 2048, 4136, (64, 64), 20)],
-                         ids=["light-tail-tiles", "split-tail"])
+@pytest.mark.parametrize("dim,ffn,S,image,valid", [(4096, 1024, 4160, (64, 64), 40), (1024, 2048, 4136, (64, 64), 20),
+                                                      (1024, 2048, 3112, (48, 64), 20)],
+                         ids=["light-tail-tiles", "light-tail-partial-round", "split-tail"])
 @pytest.mark.parametrize("dt", [E.FP16, E.BF16], ids=lambda d: NAMES[d])
 def test_qk_rounding_orders(ctx, dt, dim, ffn, S, image, valid):
     # 16-bit blocks normalise and rotate Q and K from the QKV GEMM's FP32 accumulators
     # (ERNIE_QK_ROUND_FUSED, the default); ERNIE_QK_ROUND_STORAGE first rounds the
     # projections to the storage dtype, as the reference graph does (gemm_0/gemm_1 ->
     # rmsn_9/rmsn_10). At 4160 tokens and width 4096 the Q/K/V GEMM finishes its 64 tail
-    # rows in light tiles; at width 1024 and 4136 tokens (192 full tiles) in a split tail
-    # row, whose rows take the storage order in both modes. (GEMMs of at most 128 tiles
+    # rows in light tiles, and so it does at width 1024 and 4136 tokens (192 full tiles,
+    # three quarters of a round); at 3112 tokens (144) in a split tail row, whose rows
+    # take the storage order in both modes. (GEMMs of at most 128 tiles
     # split every tile along K and so always take the storage order.) The two orders
     # differ by one rounding of Q and K: their block outputs are held to each other by the
     # reference's block gate for the dtype and by NRMSE <= 1e-3 (FP16) / 8e-3 (BF16), an
     # eighth and a quarter of that gate, and to the oracle by the gate where the oracle
-    # runs (the narrower case).
+    # runs (the narrower cases).
     w = small_block(dim=dim, ffn=ffn, seed=15)
     x, mods, cos, sin, mask = small_inputs(S=S, dim=dim, image=image, valid=valid, seed=16)
     ctx.block_upload(8, w, dim, ffn, dt)

@@ -110,8 +110,9 @@ def test_text_block_full_width_against_oracle(ctx, full_text_block, dt, S):
 
 @pytest.mark.parametrize("dt", ALL_DT, ids=lambda d: NAMES[d])
 def test_text_block_ragged_tiles_against_oracle(ctx, dt):
-    # 300 tokens: a partial 256-row GEMM tile (split-K tail) and a partial 128-query
-    # attention tile (key-range split), at a narrower width.
+    # 300 tokens: a partial 256-row GEMM tile (K splits in the 16-bit o_proj and down GEMMs;
+    # the two of K = 512 are too short for one) and a partial 128-query attention tile
+    # (key-range split), at a narrower width.
     hidden, heads, kv, ffn, S = 512, 8, 2, 1024, 300
     w = small_text_block(seed=44, hidden=hidden, heads=heads, kv_heads=kv, ffn=ffn)
     ctx.text_block_upload(4, w, hidden, heads, kv, ffn, dt)

@@ -442,9 +442,10 @@ int block_workspace(ernie_hip_ctx* ctx, int S, int dim, int ffn, int dtype, Bloc
     return ERNIE_OK;
 }
 
-// Split-K scratch of the block GEMMs: the tail row of tiles (S % 256 rows) or, for a
-// GEMM with too few tiles for the CUs, every tile: at most 256 items of up to 256 x 256
-// FP32 partials.
+// Split-K scratch of the GEMMs: the tail row of tiles (S % 256 rows) or, for a GEMM with too
+// few tiles for the CUs, every tile: at most 256 items of up to 320 x 256 FP32 partials; or
+// a tail row and up to 256 items of 256 x 256 of a partial last round; or 128 x 128 parts of
+// FP32 tiles. A launch takes no more parts than fit.
 constexpr int kSplitItems = 256;
 
 // The same buffer also holds the attention key-range parts of a partial last query

@@ -108,9 +108,11 @@ def test_gemm_last_rows_of_a_nearly_full_tile(ctx, dt, m, n, k):
     assert g["passed"], g
 
 
-@pytest.mark.parametrize("m,n,k,ldc", [(1, 5, 16, 7), (127, 132, 48, 132), (129, 128, 80, 128), (260, 260, 1040, 261)])
+@pytest.mark.parametrize("m,n,k,ldc", [(1, 5, 16, 7), (260, 260, 16, 260), (127, 132, 48, 132), (129, 128, 80, 128),
+                                       (260, 260, 1040, 261)])
 def test_gemm_fp32_split_products(ctx, m, n, k, ldc):
-    # Tile edges, K steps of 16 past a multiple of 32, unaligned output rows. The three
+    # Tile edges, K steps of 16 past a multiple of 32, unaligned output rows (K = 16: on the
+    # FP32 matrix cores, without a split). The three
     # parts are exact and the products left out below 2^-24 of a product, so the error is
     # that of k FP32 roundings: k 2^-24 of sum |a| |w|. In the 2-norm 2e-8 to 2e-7 of the
     # result were measured; without one of the six partial products it is 1.8e-6 and more.
